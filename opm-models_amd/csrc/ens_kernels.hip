@@ -127,10 +127,10 @@ __global__ __launch_bounds__(kT) void k_e_xdot(const EnsInst* __restrict__ insts
     ExactAcc* acc = accAll + 2 * it.x;
     flushLimbs(sAcc, NACC, sMeta, acc);
     if (!lastToFinish(tickets + it.x, it.z, sMeta)) return;
-    __shared__ long long sD[kAccLimbs];
-    const double s0 = finishExact(&acc[0], sD, sMeta);
-    const double s1 = NACC == 2 ? finishExact(&acc[1], sD, sMeta) : 0.0;
+    double s[2];
+    finishSums<NACC>(acc, s);
     if (threadIdx.x != 0) return;
+    const double s0 = s[0], s1 = s[1];
     KrylovScalars* ks = ksAll + it.x;
     // failures carry the iteration's tag (tag_base = 2 it, advanced on the device)
     const int tag = ks->tag_base + tagOff;

@@ -134,6 +134,42 @@ __host__ __device__ inline double exactRound(long long* d, int lo, int hi, unsig
 }
 
 #ifdef __HIPCC__
+// Reductions over a wave by DPP moves (row shifts, then the two row
+// broadcasts): the result is lane 63's.  Absent lanes contribute zero bits.
+template <int Ctrl, int RowMask>
+__device__ __forceinline__ unsigned dppMove(unsigned x)
+{
+    return (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, Ctrl, RowMask, 0xf, false);
+}
+template <int Ctrl, int RowMask>
+__device__ __forceinline__ double dppMove(double x)
+{
+    return __hiloint2double((int)dppMove<Ctrl, RowMask>((unsigned)__double2hiint(x)),
+                            (int)dppMove<Ctrl, RowMask>((unsigned)__double2loint(x)));
+}
+// the wave's sum in every lane; for sums that are exact in every order
+__device__ __forceinline__ double waveSumExact(double v)
+{
+    v += dppMove<0x111, 0xf>(v);     // row_shr:1, 2, 4, 8
+    v += dppMove<0x112, 0xf>(v);
+    v += dppMove<0x114, 0xf>(v);
+    v += dppMove<0x118, 0xf>(v);
+    v += dppMove<0x142, 0xa>(v);     // row_bcast:15 into rows 1 and 3
+    v += dppMove<0x143, 0xc>(v);     // row_bcast:31 into rows 2 and 3
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 63),
+                            __builtin_amdgcn_readlane(__double2loint(v), 63));
+}
+__device__ __forceinline__ unsigned waveMaxU(unsigned v)
+{
+    v = max(v, dppMove<0x111, 0xf>(v));
+    v = max(v, dppMove<0x112, 0xf>(v));
+    v = max(v, dppMove<0x114, 0xf>(v));
+    v = max(v, dppMove<0x118, 0xf>(v));
+    v = max(v, dppMove<0x142, 0xa>(v));
+    v = max(v, dppMove<0x143, 0xc>(v));
+    return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
+
 constexpr int kWindow = 8;      // limbs of a wave's register window (256 bits)
 
 // Adds U products per lane of a wave to the workgroup's limbs sAcc (LDS,
@@ -202,13 +238,14 @@ __device__ __forceinline__ void addToLimbs(double v, unsigned long long* sAcc, u
 template <int U>
 __device__ __forceinline__ void accumulateBands(const double (&p)[U], unsigned long long* sAcc, unsigned& flags)
 {
-    int emax = -2000;
+    unsigned be = 0u;            // the largest biased exponent of a finite product
 #pragma unroll
-    for (int u = 0; u < U; ++u)
-        if (p[u] != 0.0 && isfinite(p[u])) emax = max(emax, ilogb(p[u]));
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) emax = max(emax, __shfl_xor(emax, o, 64));
-    if (emax < -700 || emax > 1000) {            // no finite nonzero product, or extreme ones
+    for (int u = 0; u < U; ++u) {
+        const unsigned e = ((unsigned)__double2hiint(p[u]) >> 20) & 0x7ffu;
+        be = max(be, e == 0x7ffu ? 0u : e);
+    }
+    be = waveMaxU(be);
+    if (be < 1023u - 700u || be > 1023u + 1000u) {     // no finite nonzero product, or extreme ones
         accumulateWave<U>(p, sAcc, flags);
         return;
     }
@@ -216,7 +253,7 @@ __device__ __forceinline__ void accumulateBands(const double (&p)[U], unsigned l
     double S[kBands];
 #pragma unroll
     for (int i = 0; i < kBands; ++i) S[i] = 0.0;
-    const double sigma0 = ldexp(1.0, emax + 10);
+    const double sigma0 = __hiloint2double((int)((be + 10u) << 20), 0);     // 2^(e_max + 10)
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         if (!isfinite(p[u])) { addToLimbs(p[u], sAcc, flags); continue; }
@@ -231,9 +268,7 @@ __device__ __forceinline__ void accumulateBands(const double (&p)[U], unsigned l
         if (r != 0.0) addToLimbs(r, sAcc, flags);
     }
 #pragma unroll
-    for (int i = 0; i < kBands; ++i)
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) S[i] += __shfl_xor(S[i], o, 64);
+    for (int i = 0; i < kBands; ++i) S[i] = waveSumExact(S[i]);
     const int lane = (int)(threadIdx.x & 63u);
     if (lane < kBands) {
         double v = 0.0;
@@ -284,30 +319,133 @@ __device__ __forceinline__ bool lastToFinish(unsigned* ticket, int nBlocks, unsi
     return sMeta[1] != 0u;
 }
 
-// In the last workgroup: the rounded value of the device accumulator g, which
-// is cleared for the next use.  sD: LDS of kAccLimbs long longs.
-__device__ __forceinline__ double finishExact(ExactAcc* g, long long* sD, unsigned* sMeta)
+// The same for a whole grid: many workgroups meet in kFinishGroups groups
+// first, whose tickets lie in lines of their own.  Atomics on one word pass at
+// about 13 ns each, so 256 workgroups on one ticket take 3.3 us; the groups'
+// second round trip takes 1 us, which fewer than 64 workgroups would not win
+// back.
+constexpr int kFinishGroups = 16, kFinishFlat = 64;
+struct alignas(128) FinishTicket {
+    unsigned n;
+};
+// tickets: kFinishGroups + 1, the last one the groups' own
+__device__ __forceinline__ bool lastOfGrid(FinishTicket* tickets, unsigned* sMeta)
 {
-    if (threadIdx.x < kAccLimbs) {
-        const unsigned long long v =
-            __hip_atomic_load(&g->limb[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        sD[threadIdx.x] = (long long)v;
-        if (v) __hip_atomic_store(&g->limb[threadIdx.x], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int nb = (int)gridDim.x, G = nb > kFinishFlat ? kFinishGroups : 1, g = (int)blockIdx.x % G;
+    if (!lastToFinish(&tickets[g].n, (nb - g + G - 1) / G, sMeta)) return false;
+    return G == 1 || lastToFinish(&tickets[kFinishGroups].n, G, sMeta);
+}
+
+// exactRound by one wave: lane j holds limb j as a signed integer, and limbs
+// 62 and up are zero.  Every lane gets the value.
+__device__ __forceinline__ double waveRound(long long limb, unsigned flags)
+{
+    if ((flags & 1u) || (flags & 6u) == 6u) return __longlong_as_double(0x7FF8000000000000ll);
+    if (flags & 2u) return __longlong_as_double(0x7FF0000000000000ll);
+    if (flags & 4u) return __longlong_as_double((long long)0xFFF0000000000000ull);
+    const unsigned long long nz = __ballot(limb != 0);
+    if (!nz) return 0.0;
+    const int lane = (int)(threadIdx.x & 63u);
+    const int lo = __builtin_ctzll(nz), top = 64 - __builtin_clzll(nz);      // one above the last nonzero limb
+    unsigned dg = 0u;               // lane j: digit j of the magnitude
+    bool neg = false;
+    for (int pass = 0; pass < 2; ++pass) {
+        long long carry = 0;
+        for (int j = lo; j <= top; ++j) {
+            const unsigned wl = (unsigned)__builtin_amdgcn_readlane((int)limb, j);
+            const int wh = __builtin_amdgcn_readlane((int)(limb >> 32), j);
+            const long long t = (long long)(((unsigned long long)(unsigned)wh << 32) | wl) + carry;
+            dg = lane == j ? (unsigned)t : dg;
+            carry = t >> 32;
+        }
+        if (carry >= 0) break;
+        neg = true;                 // the magnitude: the digits of the negated limbs
+        limb = -limb;
     }
-    if (threadIdx.x == 0) {
-        sMeta[2] = __hip_atomic_load(&g->flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (sMeta[2]) __hip_atomic_store(&g->flags, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    __syncthreads();
-    __shared__ double sR;
-    if (threadIdx.x == 0) {
+    const unsigned long long dz = __ballot(dg != 0u);
+    if (!dz) return 0.0;
+    const int h = 63 - __builtin_clzll(dz);
+    auto dig = [&](int j) -> unsigned long long {
+        return j < 0 ? 0ull : (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)dg, j);
+    };
+    const unsigned long long sgn = neg ? (1ull << 63) : 0ull;
+    const unsigned long long hiw = dig(h), midw = dig(h - 1), low = dig(h - 2);
+    const int lz = __builtin_clz((unsigned)hiw);
+    int b = 32 * h + 31 - lz;       // leading bit, in units of 2^-1074
+    if (b < 53)                     // subnormal or smallest normal: exact
+        return __longlong_as_double((long long)(sgn | (dig(1) << 32) | dig(0)));
+    const int s = 32 - lz;          // bits of digit h - 2 below the window of 64
+    const unsigned long long w = (hiw << (64 - s)) | (midw << (32 - s)) | (low >> s);
+    const bool below = h > 2 && (dz & ((1ull << (h - 2)) - 1ull)) != 0ull;
+    const bool sticky = (low & ((1ull << s) - 1ull)) != 0ull || below;
+    unsigned long long mant = w >> 11;
+    if (((w >> 10) & 1ull) && ((w & 0x3ffull) != 0ull || sticky || (mant & 1ull))) ++mant;
+    if (mant >> 53) { mant >>= 1; ++b; }
+    const int biased = b - 51;
+    if (biased >= 2047) return __longlong_as_double((long long)(sgn | 0x7FF0000000000000ull));
+    return __longlong_as_double((long long)(sgn | ((unsigned long long)biased << 52) | (mant & 0xFFFFFFFFFFFFFull)));
+}
+
+// The rounded value of an accumulator in one wave's registers: v0 limb
+// `lane`, v1 limb 64 + lane (zero where there is none).
+__device__ __forceinline__ double roundLimbs(unsigned long long v0, unsigned long long v1, unsigned flags,
+                                             long long* sD)
+{
+    const int lane = (int)(threadIdx.x & 63u);
+    if (__ballot(v1 != 0ull || (lane >= 62 && v0 != 0ull)) == 0ull) return waveRound((long long)v0, flags);
+    // products of 2^910 and more: one thread over LDS
+    sD[lane] = (long long)v0;
+    if (lane + 64 < kAccLimbs) sD[lane + 64] = (long long)v1;
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    double r = 0.0;
+    if (lane == 0) {
         int lo = kAccLimbs, hi = -1;
         for (int t = 0; t < kAccLimbs; ++t)
             if (sD[t]) { if (lo == kAccLimbs) lo = t; hi = t; }
-        sR = exactRound(sD, lo, hi, sMeta[2]);
+        r = exactRound(sD, lo, hi, flags);
     }
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(r)),
+                            __builtin_amdgcn_readfirstlane(__double2loint(r)));
+}
+
+// In one wave of the last workgroup: the rounded value of the device
+// accumulator g, which is cleared for the next use; every lane gets it.  sD:
+// LDS of kAccLimbs long longs of this wave's own.  The chain of carries over
+// the limbs bounds it: it runs through readlane and scalar adds instead of one
+// thread's LDS accesses, 0.6 us instead of 3.0 us per sum.
+__device__ __forceinline__ double finishExact(ExactAcc* g, long long* sD)
+{
+    const int lane = (int)(threadIdx.x & 63u);
+    const bool two = lane + 64 < kAccLimbs;
+    const unsigned long long v0 = __hip_atomic_load(&g->limb[lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned long long v1 =
+        two ? __hip_atomic_load(&g->limb[lane + 64], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
+    const unsigned flags = (unsigned)__builtin_amdgcn_readfirstlane(
+        (int)__hip_atomic_load(&g->flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    if (v0) __hip_atomic_store(&g->limb[lane], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (v1) __hip_atomic_store(&g->limb[lane + 64], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (flags && lane == 0) __hip_atomic_store(&g->flags, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return roundLimbs(v0, v1, flags, sD);
+}
+
+// In the last workgroup (at least NACC waves): the sums g[0..NACC) in every
+// thread of wave 0; one wave per sum.
+template <int NACC>
+__device__ __forceinline__ void finishSums(ExactAcc* g, double (&sum)[2])
+{
+    __shared__ long long sD[NACC * kAccLimbs];
+    __shared__ double sR[NACC];
+    const int w = (int)(threadIdx.x >> 6);
+    sum[0] = sum[1] = 0.0;
+    if (w < NACC) {
+        sum[0] = finishExact(g + w, sD + w * kAccLimbs);
+        sR[w] = sum[0];
+    }
+    if (NACC == 1) return;
     __syncthreads();
-    return sR;
+    sum[0] = sR[0];
+    sum[1] = sR[NACC - 1];
 }
 #endif
 

@@ -1072,7 +1072,7 @@ int BiCGStabBackend::bicgstab(const S* A, const S* lu, const void* dinv, const S
             m_.timer.end(s);
         }
         launchDotFinal<S>(m, b, v, m_.dots.p, ks_.p, 1, 0, s);
-        launchUpdateXR<S>(m, y, v, x, r, m_.partial.p, ks_.p, s);
+        launchUpdateXR<S>(m, y, v, x, r, m_.dots.p, ks_.p, s);
     };
     // second half: z = M^-1 r, y = A z, omega, x/r update, next tag base
     auto secondHalf = [&]() {
@@ -1083,13 +1083,13 @@ int BiCGStabBackend::bicgstab(const S* A, const S* lu, const void* dinv, const S
             m_.timer.end(s);
         }
         launchDot2Final<S>(m, y, r, m_.dots.p, ks_.p, 1, s);
-        launchUpdateXR2<S>(m, z, y, x, r, m_.partial.p, ks_.p, 1, 2, s);
+        launchUpdateXR2<S>(m, z, y, x, r, m_.dots.p, ks_.p, 1, 2, s);
     };
 
     IterGraphs* gr = nullptr;
     if (prm_.graph) {
         gr = &graphs_[sizeof(S) == 4 ? 1 : 0];
-        const std::array<const void*, 12> key = {A, lu, dinv, b, x, r, p, v, y, z, m_.partial.p, ks_.p};
+        const std::array<const void*, 12> key = {A, lu, dinv, b, x, r, p, v, y, z, m_.dots.p, ks_.p};
         // the tiled ILU's device descriptors of both applications must be
         // resident before a capture (an upload cannot be recorded); a cache
         // turnover between the two primes is followed by one more pass

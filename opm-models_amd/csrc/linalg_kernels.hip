@@ -642,46 +642,75 @@ __device__ __forceinline__ void dotEpilogue(int mode, double s0, double s1, Kryl
     }
 }
 
-// NACC = 1: sum a.b;  NACC = 2: sums a.b and a.c
+// 16 bytes of a vector at the alignment of its scalar (a caller's own vector
+// may start at any element)
+template <class S>
+struct __attribute__((packed, aligned(sizeof(S)))) Vec16 {
+    static constexpr int kN = 16 / (int)sizeof(S);
+    S x[kN];
+};
+
+// NACC = 1: sum a.b;  NACC = 2: sums a.a and a.b
+// Small products are bounded by latency (the launch, one pass, the limbs'
+// and the ticket's atomics, the rounding), large ones by the loads: each wave
+// takes kDotUnroll * 64 consecutive entries per pass in 16-byte loads and
+// issues the next pass's before it splits this one's products.  FP64, us by
+// entries (before: 8-byte loads, one thread rounding):
+//   NACC 1: 1440 5.4 (8.2), 400k 6.8 (9.9), 1.5M 9.3 (13.4), 6M 20.5 (36.6);
+//   NACC 2: 1440 7.2 (13.1), 400k 8.8 (15.3), 1.5M 13.2 (23.0).
 template <class S, int NACC>
 __global__ __launch_bounds__(kDotThreads) void k_xdot(long m, const S* __restrict__ a, const S* __restrict__ b,
-    const S* __restrict__ c, DotScratch* __restrict__ sc, KrylovScalars* ks, int mode, double eps, int tagOff,
-    double* out)
+    DotScratch* __restrict__ sc, KrylovScalars* ks, int mode, double eps, int tagOff, double* out)
 {
     if (ks && !ks->run) return;
-    constexpr int nw = kDotThreads / 64;
+    constexpr int nw = kDotThreads / 64, V = Vec16<S>::kN;
     __shared__ unsigned long long sAcc[NACC * kAccLimbs];
     __shared__ unsigned sMeta[5];
     clearLimbs(sAcc, NACC, sMeta);
     __syncthreads();
     const int lane = (int)(threadIdx.x & 63u);
-    const long wavesTotal = (long)gridDim.x * nw;
+    S xa[kDotUnroll], xb[kDotUnroll];
+    auto load = [&](long base) {
+#pragma unroll
+        for (int u = 0; u < kDotUnroll; u += V) {
+            const long i = base + 64L * u + (long)V * lane;
+            if (i + V <= m) {
+                const Vec16<S> va = *reinterpret_cast<const Vec16<S>*>(a + i);
+                const Vec16<S> vb = *reinterpret_cast<const Vec16<S>*>(b + i);
+#pragma unroll
+                for (int q = 0; q < V; ++q) { xa[u + q] = va.x[q]; xb[u + q] = vb.x[q]; }
+            } else {
+#pragma unroll
+                for (int q = 0; q < V; ++q) {
+                    xa[u + q] = i + q < m ? a[i + q] : S(0);
+                    xb[u + q] = i + q < m ? b[i + q] : S(0);
+                }
+            }
+        }
+    };
     unsigned fl0 = 0u, fl1 = 0u;
-    // each wave takes kDotUnroll * 64 consecutive entries per pass (a uniform loop)
-    for (long w = (long)blockIdx.x * nw + (long)(threadIdx.x >> 6); w * (kDotUnroll * 64) < m; w += wavesTotal) {
-        const long base = w * (kDotUnroll * 64) + lane;
+    const long stride = (long)gridDim.x * nw * (kDotUnroll * 64);
+    long base = ((long)blockIdx.x * nw + (long)(threadIdx.x >> 6)) * (kDotUnroll * 64);
+    if (base < m) load(base);
+    for (; base < m; base += stride) {      // a uniform loop in each wave
         double v0[kDotUnroll], v1[kDotUnroll];
 #pragma unroll
         for (int u = 0; u < kDotUnroll; ++u) {
-            const long i = base + 64L * u;
-            v0[u] = 0.0; v1[u] = 0.0;
-            if (i < m) {
-                const double ai = (double)a[i];
-                v0[u] = ai * (double)b[i];
-                if (NACC == 2) v1[u] = ai * (double)c[i];
-            }
+            const double ai = (double)xa[u];
+            v0[u] = ai * (NACC == 2 ? ai : (double)xb[u]);
+            if (NACC == 2) v1[u] = ai * (double)xb[u];
         }
+        if (base + stride < m) load(base + stride);
         accumulateBands<kDotUnroll>(v0, sAcc, fl0);
         if (NACC == 2) accumulateBands<kDotUnroll>(v1, sAcc + kAccLimbs, fl1);
     }
     if (fl0 | fl1) atomicOr(&sMeta[0], fl0 | (fl1 << 3));
     __syncthreads();
     flushLimbs(sAcc, NACC, sMeta, sc->acc);
-    if (!lastToFinish(&sc->ticket, (int)gridDim.x, sMeta)) return;
-    __shared__ long long sD[kAccLimbs];
-    const double s0 = finishExact(&sc->acc[0], sD, sMeta);
-    const double s1 = NACC == 2 ? finishExact(&sc->acc[1], sD, sMeta) : 0.0;
-    if (threadIdx.x == 0) dotEpilogue(mode, s0, s1, ks, eps, tagOff, out);
+    if (!lastToFinish(&sc->ticket.n, (int)gridDim.x, sMeta)) return;
+    double s[2];
+    finishSums<NACC>(sc->acc, s);
+    if (threadIdx.x == 0) dotEpilogue(mode, s[0], s[1], ks, eps, tagOff, out);
 }
 
 template <class S>
@@ -689,7 +718,7 @@ void launchDotFinal(long m, const S* x, const S* y, DotScratch* sc, KrylovScalar
                     hipStream_t st)
 {
     const double eps = (double)std::numeric_limits<S>::min() * 1e10;
-    hipLaunchKernelGGL((k_xdot<S, 1>), dim3(dotBlocks(m)), dim3(kDotThreads), 0, st, m, x, y, y, sc, ks,
+    hipLaunchKernelGGL((k_xdot<S, 1>), dim3(dotBlocks(m)), dim3(kDotThreads), 0, st, m, x, y, sc, ks,
                        op == 0 ? (int)kDotRho : (int)kDotAlpha, eps, tagOff, (double*)nullptr);
 }
 template void launchDotFinal<double>(long, const double*, const double*, DotScratch*, KrylovScalars*, int, int, hipStream_t);
@@ -697,73 +726,18 @@ template void launchDotFinal<float>(long, const float*, const float*, DotScratch
 
 void launchScalarProduct(long m, const double* x, const double* y, DotScratch* sc, double* out, hipStream_t st)
 {
-    hipLaunchKernelGGL((k_xdot<double, 1>), dim3(dotBlocks(m)), dim3(kDotThreads), 0, st, m, x, y, y, sc,
+    hipLaunchKernelGGL((k_xdot<double, 1>), dim3(dotBlocks(m)), dim3(kDotThreads), 0, st, m, x, y, sc,
                        (KrylovScalars*)nullptr, (int)kDotValue, 0.0, 0, out);
 }
 
-// p = r + (-beta) * (v*omega - p)   (bicgstabsolver.hh:211-222)
-template <class S>
-__global__ void k_update_p(long m, const S* __restrict__ r, const S* __restrict__ v, S* __restrict__ p,
-                           const KrylovScalars* __restrict__ ks)
+// the test after the first half of iteration tag_base / 2 (bicgstabsolver.hh:
+// 252-273) with the outcome of the previous second half (:286-318), in the
+// order of the host loop; once it ends the solve, the queued kernels of
+// the next iteration return at once
+__device__ __forceinline__ void criterion(double mx, bool change, KrylovScalars* ks)
 {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= m || !ks->run) return;
-    const S omega = (S)ks->omega, beta = (S)ks->beta;
-    S tmp = v[i];
-    tmp *= omega;
-    tmp -= p[i];
-    tmp *= -beta;
-    S pn = r[i];
-    pn += tmp;
-    p[i] = pn;
-}
-template <class S>
-void launchUpdateP(long m, const S* r, const S* v, S* p, const KrylovScalars* ks, hipStream_t st)
-{
-    hipLaunchKernelGGL((k_update_p<S>), dim3((m + 255) / 256), dim3(256), 0, st, m, r, v, p, ks);
-}
-template void launchUpdateP<double>(long, const double*, const double*, double*, const KrylovScalars*, hipStream_t);
-template void launchUpdateP<float>(long, const float*, const float*, float*, const KrylovScalars*, hipStream_t);
-
-// x = x + alpha*y; r -= alpha*v; partials: max|r|, count(y != 0)  (:240-253)
-template <class S>
-__global__ __launch_bounds__(kRedThreads) void k_update_xr(long m, const S* __restrict__ y, const S* __restrict__ v,
-    S* __restrict__ x, S* __restrict__ r, double* __restrict__ part, const KrylovScalars* __restrict__ ks)
-{
-    if (!ks->run) return;
-    const S alpha = (S)ks->alpha;
-    double mx = 0.0, nz = 0.0;
-    for (long i = (long)blockIdx.x * kRedThreads + threadIdx.x; i < m; i += (long)kRedBlocks * kRedThreads) {
-        const S yi = y[i];
-        S tmp = yi;
-        tmp *= alpha;
-        tmp += x[i];
-        x[i] = tmp;
-        tmp = v[i];
-        tmp *= alpha;
-        S ri = r[i];
-        ri -= tmp;
-        r[i] = ri;
-        mx = fmax(mx, fabs((double)ri));
-        if (yi != S(0)) nz = 1.0;
-    }
-    mx = blockReduce<true>(mx);
-    nz = blockReduce<true>(nz);
-    if (threadIdx.x == 0) { part[blockIdx.x] = mx; part[kRedBlocks + blockIdx.x] = nz; }
-}
-
-__global__ __launch_bounds__(kRedThreads) void k_crit_final(const double* __restrict__ part, KrylovScalars* ks)
-{
-    if (!ks->run) return;
-    const double mx = finalReduce<true>(part);
-    const double nz = finalReduce<true>(part + kRedBlocks);
-    if (threadIdx.x != 0) return;
     ks->resnorm = mx;
-    ks->stag_half = (nz == 0.0) ? 1 : 0;
-    // the test after the first half of iteration tag_base / 2 (bicgstabsolver.hh:
-    // 252-273) with the outcome of the previous second half (:286-318), in the
-    // order of the host loop; once it ends the solve, the queued kernels of
-    // the next iteration return at once
+    ks->stag_half = change ? 0 : 1;
     const int tag = ks->tag_base;
     int rc = -1, back = 0;
     if (tag > 0 && ks->fail_code && ks->fail_tag == tag - 1) { rc = 2; back = 1; }
@@ -778,61 +752,206 @@ __global__ __launch_bounds__(kRedThreads) void k_crit_final(const double* __rest
     }
 }
 
-template <class S>
-void launchUpdateXR(long m, const S* y, const S* v, S* x, S* r, double* partial, KrylovScalars* ks, hipStream_t st)
+// The iterate's updates: one element-wise pass each, bounded by the memory
+// (48 bytes an FP64 entry) or, on small systems, by the launch.  The maximum
+// and the change indicator of the workgroups are joined, and the test
+// evaluated, by the workgroup that finishes last: no second launch for them.
+constexpr int kUpdThreads = 1024;
+constexpr int kUpdBlocks = kDotMaxBlocks;     // one workgroup per CU
+
+inline int updateBlocks(long m, int perThread)
 {
-    hipLaunchKernelGGL((k_update_xr<S>), dim3(kRedBlocks), dim3(kRedThreads), 0, st, m, y, v, x, r, partial, ks);
-    hipLaunchKernelGGL(k_crit_final, dim3(1), dim3(kRedThreads), 0, st, partial, ks);
+    const long per = (long)perThread * kUpdThreads;
+    return (int)std::max(1L, std::min<long>(kUpdBlocks, (m + per - 1) / per));
 }
-template void launchUpdateXR<double>(long, const double*, const double*, double*, double*, double*, KrylovScalars*, hipStream_t);
-template void launchUpdateXR<float>(long, const float*, const float*, float*, float*, double*, KrylovScalars*, hipStream_t);
+
+// f(i0, n): entries i0 .. i0 + n - 1 (n <= V, a compile-time V for full ones)
+template <int V, class F>
+__device__ __forceinline__ void forEntries(long m, F f)
+{
+    const long step = (long)gridDim.x * kUpdThreads * V;
+    for (long i = ((long)blockIdx.x * kUpdThreads + threadIdx.x) * V; i < m; i += step) f(i, (int)min((long)V, m - i));
+}
+
+template <int V, class S>
+__device__ __forceinline__ void loadEntries(const S* p, long i, int n, S (&x)[V])
+{
+    if (n == V) {
+        const Vec16<S> t = *reinterpret_cast<const Vec16<S>*>(p + i);
+#pragma unroll
+        for (int q = 0; q < V; ++q) x[q] = t.x[q];
+    } else {
+#pragma unroll
+        for (int q = 0; q < V; ++q) x[q] = q < n ? p[i + q] : S(0);
+    }
+}
+template <int V, class S>
+__device__ __forceinline__ void storeEntries(S* p, long i, int n, const S (&x)[V])
+{
+    if (n == V) {
+        Vec16<S> t;
+#pragma unroll
+        for (int q = 0; q < V; ++q) t.x[q] = x[q];
+        *reinterpret_cast<Vec16<S>*>(p + i) = t;
+    } else {
+#pragma unroll
+        for (int q = 0; q < V; ++q)
+            if (q < n) p[i + q] = x[q];
+    }
+}
+
+// p = r + (-beta) * (v*omega - p)   (bicgstabsolver.hh:211-222)
+template <class S>
+__global__ __launch_bounds__(kUpdThreads) void k_update_p(long m, const S* __restrict__ r, const S* __restrict__ v,
+    S* __restrict__ p, const KrylovScalars* __restrict__ ks)
+{
+    if (!ks->run) return;
+    constexpr int V = Vec16<S>::kN;
+    const S omega = (S)ks->omega, beta = (S)ks->beta;
+    forEntries<V>(m, [&](long i, int n) {
+        S rv[V], vv[V], pv[V];
+        loadEntries<V>(v, i, n, vv); loadEntries<V>(p, i, n, pv); loadEntries<V>(r, i, n, rv);
+#pragma unroll
+        for (int q = 0; q < V; ++q) {
+            S tmp = vv[q];
+            tmp *= omega;
+            tmp -= pv[q];
+            tmp *= -beta;
+            S pn = rv[q];
+            pn += tmp;
+            pv[q] = pn;
+        }
+        storeEntries<V>(p, i, n, pv);
+    });
+}
+template <class S>
+void launchUpdateP(long m, const S* r, const S* v, S* p, const KrylovScalars* ks, hipStream_t st)
+{
+    hipLaunchKernelGGL((k_update_p<S>), dim3(updateBlocks(m, Vec16<S>::kN)), dim3(kUpdThreads), 0, st, m, r, v, p, ks);
+}
+template void launchUpdateP<double>(long, const double*, const double*, double*, const KrylovScalars*, hipStream_t);
+template void launchUpdateP<float>(long, const float*, const float*, float*, const KrylovScalars*, hipStream_t);
+
+// Joins the workgroups' maximum and change indicator; true in thread 0 of the
+// last workgroup, which then has both over all entries.
+__device__ __forceinline__ bool joinUpdate(DotScratch* sc, double& mx, bool& change)
+{
+    constexpr int nw = kUpdThreads / 64;
+    __shared__ double sMx[nw];
+    __shared__ unsigned sMeta[2], sAny[nw];
+    const int lane = (int)(threadIdx.x & 63u), w = (int)(threadIdx.x >> 6);
+    mx = waveMax(mx);
+    const bool any = __ballot(change) != 0ull;
+    if (lane == 0) { sMx[w] = mx; sAny[w] = any ? 1u : 0u; }
+    __syncthreads();
+    if (w == 0) {
+        mx = waveMax(lane < nw ? sMx[lane] : 0.0);
+        change = __ballot(lane < nw && sAny[lane]) != 0ull;
+        if (gridDim.x == 1) return lane == 0;
+        if (lane == 0) {
+            __hip_atomic_store(&sc->blockMax[blockIdx.x], mx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&sc->blockAny[blockIdx.x], change ? 1u : 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+    if (gridDim.x == 1 || !lastOfGrid(sc->updTicket, sMeta) || w != 0) return false;
+    mx = 0.0;
+    unsigned a = 0u;
+    for (int k = lane; k < (int)gridDim.x; k += 64) {
+        mx = fmax(mx, __hip_atomic_load(&sc->blockMax[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        a |= __hip_atomic_load(&sc->blockAny[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    mx = waveMax(mx);
+    change = __ballot(a != 0u) != 0ull;
+    return lane == 0;
+}
+
+// x = x + alpha*y; r -= alpha*v; max|r|, whether y != 0 anywhere  (:240-253)
+template <class S>
+__global__ __launch_bounds__(kUpdThreads) void k_update_xr(long m, const S* __restrict__ y, const S* __restrict__ v,
+    S* __restrict__ x, S* __restrict__ r, DotScratch* __restrict__ sc, KrylovScalars* ks)
+{
+    if (!ks->run) return;
+    constexpr int V = Vec16<S>::kN;
+    const S alpha = (S)ks->alpha;
+    double mx = 0.0;
+    bool change = false;
+    forEntries<V>(m, [&](long i, int n) {
+        S yv[V], vv[V], xv[V], rv[V];
+        loadEntries<V>(y, i, n, yv); loadEntries<V>(x, i, n, xv);
+        loadEntries<V>(v, i, n, vv); loadEntries<V>(r, i, n, rv);
+#pragma unroll
+        for (int q = 0; q < V; ++q) {
+            S tmp = yv[q];
+            tmp *= alpha;
+            tmp += xv[q];
+            xv[q] = tmp;
+            tmp = vv[q];
+            tmp *= alpha;
+            rv[q] -= tmp;
+            if (q < n) {
+                mx = fmax(mx, fabs((double)rv[q]));
+                change |= yv[q] != S(0);
+            }
+        }
+        storeEntries<V>(x, i, n, xv); storeEntries<V>(r, i, n, rv);
+    });
+    if (joinUpdate(sc, mx, change)) criterion(mx, change, ks);
+}
+
+template <class S>
+void launchUpdateXR(long m, const S* y, const S* v, S* x, S* r, DotScratch* sc, KrylovScalars* ks, hipStream_t st)
+{
+    hipLaunchKernelGGL((k_update_xr<S>), dim3(updateBlocks(m, Vec16<S>::kN)), dim3(kUpdThreads), 0, st, m, y, v, x, r, sc, ks);
+}
+template void launchUpdateXR<double>(long, const double*, const double*, double*, double*, DotScratch*, KrylovScalars*, hipStream_t);
+template void launchUpdateXR<float>(long, const float*, const float*, float*, float*, DotScratch*, KrylovScalars*, hipStream_t);
 
 // <t,t> and <t,s> in one pass; omega = <t,s>/<t,t>  (:287-292)
 template <class S>
 void launchDot2Final(long m, const S* t, const S* s, DotScratch* sc, KrylovScalars* ks, int tagOff, hipStream_t st)
 {
     const double eps = (double)std::numeric_limits<S>::min() * 1e10;
-    hipLaunchKernelGGL((k_xdot<S, 2>), dim3(dotBlocks(m)), dim3(kDotThreads), 0, st, m, t, t, s, sc, ks,
+    hipLaunchKernelGGL((k_xdot<S, 2>), dim3(dotBlocks(m)), dim3(kDotThreads), 0, st, m, t, s, sc, ks,
                        (int)kDotOmega, eps, tagOff, (double*)nullptr);
 }
 template void launchDot2Final<double>(long, const double*, const double*, DotScratch*, KrylovScalars*, int, hipStream_t);
 template void launchDot2Final<float>(long, const float*, const float*, DotScratch*, KrylovScalars*, int, hipStream_t);
 
-// x += omega*z (criterion change indicator z), r += -omega*t  (:296-325)
+// x += omega*z, r += -omega*t; whether z != 0 anywhere; the iteration's end  (:296-325)
 template <class S>
-__global__ __launch_bounds__(kRedThreads) void k_update_xr2(long m, const S* __restrict__ z, const S* __restrict__ t,
-    S* __restrict__ x, S* __restrict__ r, double* __restrict__ part, const KrylovScalars* __restrict__ ks)
+__global__ __launch_bounds__(kUpdThreads) void k_update_xr2(long m, const S* __restrict__ z, const S* __restrict__ t,
+    S* __restrict__ x, S* __restrict__ r, DotScratch* __restrict__ sc, KrylovScalars* ks, int tagOff, int advance)
 {
     if (!ks->run) return;
+    constexpr int V = Vec16<S>::kN;
     const S omega = (S)ks->omega;
-    double nz = 0.0;
-    for (long i = (long)blockIdx.x * kRedThreads + threadIdx.x; i < m; i += (long)kRedBlocks * kRedThreads) {
-        const S zi = z[i];
-        x[i] += omega * zi;
-        if (zi != S(0)) nz = 1.0;
-        r[i] += -omega * t[i];
-    }
-    nz = blockReduce<true>(nz);
-    if (threadIdx.x == 0) part[blockIdx.x] = nz;
-}
-__global__ __launch_bounds__(kRedThreads) void k_stag_final(const double* __restrict__ part, KrylovScalars* ks,
-                                                            int tagOff, int advance)
-{
-    if (!ks->run) return;
-    const double nz = finalReduce<true>(part);
-    if (threadIdx.x != 0) return;
-    if (nz == 0.0 && ks->stag_full_tag < 0) ks->stag_full_tag = ks->tag_base + tagOff;
+    double mx = 0.0;
+    bool change = false;
+    forEntries<V>(m, [&](long i, int n) {
+        S zv[V], tv[V], xv[V], rv[V];
+        loadEntries<V>(z, i, n, zv); loadEntries<V>(x, i, n, xv);
+        loadEntries<V>(t, i, n, tv); loadEntries<V>(r, i, n, rv);
+#pragma unroll
+        for (int q = 0; q < V; ++q) {
+            xv[q] += omega * zv[q];
+            if (q < n) change |= zv[q] != S(0);
+            rv[q] += -omega * tv[q];
+        }
+        storeEntries<V>(x, i, n, xv); storeEntries<V>(r, i, n, rv);
+    });
+    if (!joinUpdate(sc, mx, change)) return;
+    if (!change && ks->stag_full_tag < 0) ks->stag_full_tag = ks->tag_base + tagOff;
     ks->tag_base += advance;
 }
 template <class S>
-void launchUpdateXR2(long m, const S* z, const S* t, S* x, S* r, double* partial, KrylovScalars* ks, int tagOff,
+void launchUpdateXR2(long m, const S* z, const S* t, S* x, S* r, DotScratch* sc, KrylovScalars* ks, int tagOff,
                      int advance, hipStream_t st)
 {
-    hipLaunchKernelGGL((k_update_xr2<S>), dim3(kRedBlocks), dim3(kRedThreads), 0, st, m, z, t, x, r, partial, ks);
-    hipLaunchKernelGGL(k_stag_final, dim3(1), dim3(kRedThreads), 0, st, partial, ks, tagOff, advance);
+    hipLaunchKernelGGL((k_update_xr2<S>), dim3(updateBlocks(m, Vec16<S>::kN)), dim3(kUpdThreads), 0, st, m, z, t, x, r, sc, ks,
+                       tagOff, advance);
 }
-template void launchUpdateXR2<double>(long, const double*, const double*, double*, double*, double*, KrylovScalars*, int, int, hipStream_t);
-template void launchUpdateXR2<float>(long, const float*, const float*, float*, float*, double*, KrylovScalars*, int, int, hipStream_t);
+template void launchUpdateXR2<double>(long, const double*, const double*, double*, double*, DotScratch*, KrylovScalars*, int, int, hipStream_t);
+template void launchUpdateXR2<float>(long, const float*, const float*, float*, float*, DotScratch*, KrylovScalars*, int, int, hipStream_t);
 
 // max |x| -> out (device)
 template <class S>

@@ -3,8 +3,8 @@
 // forbid hipMalloc): device inputs and output, the caller's stream, and the
 // exact accumulator in a file-scope device array instead of an allocation.
 //
-// `scratch` holds the exact sum's device accumulators and ticket (DotScratch,
-// 1.3 KiB) per GPU for the life of the process.  In host code its name is
+// `scratch` holds the exact sum's device accumulators and tickets (DotScratch,
+// 6.5 KiB) per GPU for the life of the process.  In host code its name is
 // only a stand-in; the device address of each GPU's copy is looked up once per
 // device with hipGetSymbolAddress and used for every launch.  All calls on one
 // GPU share it: calls that overlap on one GPU (two streams, two threads) race
@@ -48,11 +48,8 @@ DotScratch* scratchOnCurrentDevice()
 // workgroup of every product leaves them clear, this undoes an interrupted one
 __global__ void k_clear_scratch(DotScratch* sc)
 {
-    for (int t = (int)threadIdx.x; t < kAccLimbs; t += (int)blockDim.x) {
-        sc->acc[0].limb[t] = 0ull;
-        sc->acc[1].limb[t] = 0ull;
-    }
-    if (threadIdx.x == 0) { sc->acc[0].flags = 0u; sc->acc[1].flags = 0u; sc->ticket = 0u; }
+    unsigned long long* w = reinterpret_cast<unsigned long long*>(sc);
+    for (int t = (int)threadIdx.x; t < (int)(sizeof(DotScratch) / 8); t += (int)blockDim.x) w[t] = 0ull;
 }
 
 }  // namespace
@@ -63,7 +60,7 @@ void scalarProductNoAlloc(long m, const double* x, const double* y, double* out,
         throw std::invalid_argument("scalar product without allocation: 0 <= m < 2^28 (the accumulator's limit)");
     if (!out || (m > 0 && (!x || !y))) throw std::invalid_argument("scalar product without allocation: null pointer");
     DotScratch* sc = scratchOnCurrentDevice();
-    hipLaunchKernelGGL(k_clear_scratch, dim3(1), dim3(64), 0, st, sc);
+    hipLaunchKernelGGL(k_clear_scratch, dim3(1), dim3(1024), 0, st, sc);
     launchScalarProduct(m, x, y, sc, out, st);
     OM_HIP(hipGetLastError());
 }

@@ -266,15 +266,18 @@ template <class S> void launchExtractInvDiag(int n, int bs, const int* diag, con
 
 // BiCGStab steps (see bicgstab in host_solver.cpp for the sequence)
 // tagOff: 0 for the first half of an iteration, 1 for the second (tag = ks->tag_base + tagOff)
-// Scratch of the exact scalar products (exact_sum.h): the device
-// accumulators of up to two sums and the ticket of the workgroup that
-// finishes last (all zero between products: that workgroup clears them).
+// Scratch of the exact scalar products (exact_sum.h) and of the iterate's
+// updates: the device accumulators of up to two sums and the tickets of the
+// workgroups that finish last (zero between launches: the last workgroup
+// clears them), and the workgroups' results of an update (written before they
+// are read).
 constexpr int kDotMaxBlocks = 256;
 constexpr int kDotThreads = 512;
 struct DotScratch {
     ExactAcc acc[2];
-    unsigned int ticket;
-    unsigned int pad_[63];
+    FinishTicket ticket, updTicket[kFinishGroups + 1];
+    double blockMax[kDotMaxBlocks];
+    unsigned blockAny[kDotMaxBlocks];
 };
 enum DotMode : int { kDotRho = 0, kDotAlpha = 1, kDotOmega = 2, kDotValue = 3 };
 // one launch per product: op 0 rho_i/beta, op 1 denom/alpha
@@ -286,10 +289,10 @@ void launchScalarProduct(long m, const double* x, const double* y, DotScratch* s
 void scalarProductNoAlloc(long m, const double* x, const double* y, double* out, hipStream_t st);
 template <class S> void launchUpdateP(long m, const S* r, const S* v, S* p, const KrylovScalars* ks,
                                       hipStream_t st);
-template <class S> void launchUpdateXR(long m, const S* y, const S* v, S* x, S* r, double* partial,
+template <class S> void launchUpdateXR(long m, const S* y, const S* v, S* x, S* r, DotScratch* sc,
                                        KrylovScalars* ks, hipStream_t st);
-// the second half ends the iteration: its final kernel advances tag_base by `advance`
-template <class S> void launchUpdateXR2(long m, const S* z, const S* t, S* x, S* r, double* partial,
+// the second half ends the iteration: its last workgroup advances tag_base by `advance`
+template <class S> void launchUpdateXR2(long m, const S* z, const S* t, S* x, S* r, DotScratch* sc,
                                         KrylovScalars* ks, int tagOff, int advance, hipStream_t st);
 template <class S> void launchDot2Final(long m, const S* t, const S* s, DotScratch* sc, KrylovScalars* ks,
                                         int tagOff, hipStream_t st);
