@@ -10,6 +10,7 @@
 #include <map>
 
 #include "omodels_host.h"
+#include "small_solve.h"
 
 namespace omodels {
 
@@ -71,7 +72,7 @@ Model::Model(const omodels_blackoil_problem* p, hipStream_t s)
     nbOff.upload(topo.nbOff.data(), topo.nbOff.size(), stream);
     levels.nLevels = (int)topo.levelPtr.size() - 1;
     levels.ptrHost.assign(topo.levelPtr.begin(), topo.levelPtr.end());
-    levels.rows.upload(topo.levelRows.data(), topo.levelRows.size(), stream);
+    levels.setRows(topo.levelRows, 3, topo.rowPtr.data(), topo.diagOff.data(), stream);
     nsrc = p->n_src;
     if (nsrc > 0) {
         for (int k = 0; k < nsrc; ++k)
@@ -578,8 +579,26 @@ void Model::restoreTimeLevel()
         OM_HIP(hipMemcpyAsync(aux0.p, aux1.p, 3 * nAux * sizeof(double), hipMemcpyDeviceToDevice, stream));
 }
 
-void buildLevelSchedule(long R, const std::vector<int>& rp, const std::vector<int>& ci, LevelSchedule& L,
-                        hipStream_t s)
+void LevelSchedule::setRows(const std::vector<int>& order, int bs, const int* rp, const int* diag, hipStream_t s)
+{
+    rows.upload(order.data(), order.size(), s);
+    nChunks = 0;
+    if (!smallSystem((long)order.size(), bs)) return;
+    const int per = bs == 3 ? 16 : 32;      // rows of a wave's chunk: quads or pairs of lanes
+    std::vector<int4> t((size_t)kSlotPad * per, make_int4(-1, 0, 0, -1));
+    for (int l = 0; l < nLevels; ++l)
+        for (int k = ptrHost[l]; k < ptrHost[l + 1]; k += per, ++nChunks)
+            for (int q = 0; q < per; ++q) {
+                const int i = k + q < ptrHost[l + 1] ? order[k + q] : -1;
+                if (i < 0) t.push_back(make_int4(-1, 0, 0, l));
+                else t.push_back(make_int4(i, rp[i], (diag[i] - rp[i]) | (rp[i + 1] - 1 - diag[i]) << 16, l));
+            }
+    t.resize(t.size() + (size_t)kSlotPad * per, make_int4(-1, 0, 0, nLevels));
+    slots.upload(t.data(), t.size(), s);
+}
+
+void buildLevelSchedule(long R, int bs, const std::vector<int>& rp, const std::vector<int>& ci,
+                        const std::vector<int>& diag, LevelSchedule& L, hipStream_t s)
 {
     // lower-numbered rows coupled through an entry above the diagonal
     std::vector<std::vector<int>> upFrom(R);
@@ -602,7 +621,7 @@ void buildLevelSchedule(long R, const std::vector<int>& rp, const std::vector<in
     for (int l = 0; l < nL; ++l) L.ptrHost[l + 1] += L.ptrHost[l];
     std::vector<int> order(R), fill(L.ptrHost.begin(), L.ptrHost.end() - 1);
     for (long i = 0; i < R; ++i) order[fill[lvl[i]]++] = (int)i;
-    L.rows.upload(order.data(), order.size(), s);
+    L.setRows(order, bs, rp.data(), diag.data(), s);
 }
 
 long Model::blockOffset(long row, long col) const
@@ -668,7 +687,7 @@ void Model::setAuxiliary(int n, int nLinks, const int* row, const int* col)
         diagOff.upload(xDiagOff.data(), xDiagOff.size(), stream);
         nbOff.upload(xNbOff.data(), xNbOff.size(), stream);
         nnzb = xRowPtr[R];
-        buildLevelSchedule(R, xRowPtr, xColIdx, levels, stream);
+        buildLevelSchedule(R, 3, xRowPtr, xColIdx, xDiagOff, levels, stream);
         aux0.alloc(3 * (size_t)n); aux1.alloc(3 * (size_t)n);
         OM_HIP(hipMemsetAsync(aux0.p, 0, 3 * (size_t)n * sizeof(double), stream));
         OM_HIP(hipMemsetAsync(aux1.p, 0, 3 * (size_t)n * sizeof(double), stream));
@@ -681,7 +700,7 @@ void Model::setAuxiliary(int n, int nLinks, const int* row, const int* col)
         nnzb = topo.rowPtr[N];
         levels.nLevels = (int)topo.levelPtr.size() - 1;
         levels.ptrHost.assign(topo.levelPtr.begin(), topo.levelPtr.end());
-        levels.rows.upload(topo.levelRows.data(), topo.levelRows.size(), stream);
+        levels.setRows(topo.levelRows, 3, topo.rowPtr.data(), topo.diagOff.data(), stream);
         aux0.release(); aux1.release();
     }
     jac.release();
@@ -733,6 +752,9 @@ BiCGStabBackend::BiCGStabBackend(LinearSystem& m, const omodels_params& prm)
             tiled_ = std::make_unique<TiledIlu>(makeTileGeom(m.gx, m.gy, m.gz), m.stream, mode);
         }
     }
+    // natural-order ILU(0) on a system that one workgroup solves
+    small_ = prm_.precond == 0 && !colored_ && prm_.ilu_schedule == 0 && !prm_.autotune && !prm_.spmv_in_sweep &&
+             m.levels.nChunks > 0 && (!tiled_ || n <= kSmallTiledEntries);
     if (prm_.precond == 1) {
         if (prm_.prec_order < 0) throw std::invalid_argument("PreconditionerOrder must be >= 0");
         jacTmp_.alloc(n * (prm_.precision == 0 ? sizeof(double) : sizeof(float)));
@@ -918,8 +940,12 @@ void BiCGStabBackend::prepare(const double* hostValues, const double* hostResidu
         launchCopyConvertD<float>(bb * nnzb, A64_, luf_.p, s);
         dinv64_.alloc(bb * (size_t)N);
         m_.timer.begin(kClsIluFactor, s);
-        launchIlu0Factor<float>(N, bs, m_.rowPtr.p, m_.colIdx.p, m_.diagOff.p, luf_.p, m_.levels, fail_.p, s);
-        launchExtractInvDiag<float>(N, bs, m_.diagOff.p, luf_.p, dinv64_.p, s);
+        if (small_) {
+            launchSmallFactor<float>(N, bs, m_.levels, m_.rowPtr.p, m_.colIdx.p, m_.diagOff.p, luf_.p, dinv64_.p, fail_.p, s);
+        } else {
+            launchIlu0Factor<float>(N, bs, m_.rowPtr.p, m_.colIdx.p, m_.diagOff.p, luf_.p, m_.levels, fail_.p, s);
+            launchExtractInvDiag<float>(N, bs, m_.diagOff.p, luf_.p, dinv64_.p, s);
+        }
         m_.timer.end(s);
     } else if (amg_) {
         // the AMG hierarchy of the structured FP64 matrix
@@ -942,6 +968,8 @@ void BiCGStabBackend::prepare(const double* hostValues, const double* hostResidu
         m_.timer.begin(kClsIluFactor, s);
         if (tiled_) {
             tiled_->factor(m_.rowPtr.p, m_.diagOff.p, lu64_.p, dinv64_.p, fail_.p, s);
+        } else if (small_) {
+            launchSmallFactor<double>(N, bs, m_.levels, m_.rowPtr.p, m_.colIdx.p, m_.diagOff.p, lu64_.p, dinv64_.p, fail_.p, s);
         } else {
             launchIlu0Factor<double>(N, bs, m_.rowPtr.p, m_.colIdx.p, m_.diagOff.p, lu64_.p, m_.levels, fail_.p, s);
             launchExtractInvDiag<double>(N, bs, m_.diagOff.p, lu64_.p, dinv64_.p, s);
@@ -1027,6 +1055,19 @@ int BiCGStabBackend::bicgstab(const S* A, const S* lu, const void* dinv, const S
     S* r; S* p; S* v; S* y; S* z;
     if constexpr (sizeof(S) == 8) { r = (S*)wd_[0].p; p = (S*)wd_[1].p; v = (S*)wd_[2].p; y = (S*)wd_[3].p; z = (S*)wd_[4].p; }
     else { r = (S*)wf_[0].p; p = (S*)wf_[1].p; v = (S*)wf_[2].p; y = (S*)wf_[3].p; z = (S*)wf_[4].p; }
+    if (small_ && !m_.timer.enabled) {      // timed by class, the solve goes launch by launch
+        S* const w[4] = {r, p, v, y};
+        launchSmallBicgstab<S>(N, m_.bs, m_.levels, m_.rowPtr.p, m_.colIdx.p, A, lu, (const double*)dinv, b, x, w, tol,
+                               absTol, prm_.lin_max_error, maxIter, ks_.p, s);
+        OM_HIP(hipMemcpyAsync(ksHost_, ks_.p, sizeof(KrylovScalars), hipMemcpyDeviceToHost, s));
+        m_.sync();
+        if (ksHost_->stop_rc >= 0) {
+            *its = ksHost_->iters;
+            return ksHost_->stop_rc;
+        }
+        *its = maxIter;
+        return ksHost_->fail_code ? 2 : 1;
+    }
     OM_HIP(hipMemsetAsync(x, 0, m * sizeof(S), s));
     OM_HIP(hipMemcpyAsync(r, b, m * sizeof(S), hipMemcpyDeviceToDevice, s));
     // setInitial

@@ -119,7 +119,7 @@ LensModel::LensModel(const omodels_lens_problem* p, hipStream_t s)
     for (long I = 0; I < N; ++I) rows[fill[lev[I]]++] = (int)I;
     levels.nLevels = nLev;
     levels.ptrHost = ptr;
-    levels.rows.upload(rows.data(), rows.size(), stream);
+    levels.setRows(rows, 2, hRowPtr.data(), hDiag.data(), stream);
 
     rowPtr.upload(hRowPtr.data(), hRowPtr.size(), stream);
     colIdx.upload(hColIdx.data(), hColIdx.size(), stream);

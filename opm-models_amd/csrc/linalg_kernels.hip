@@ -12,56 +12,12 @@
 // are reproducible run to run; BiCGStab scalars stay in device memory.
 #include <hipcub/hipcub.hpp>
 
+#include "block_ops.h"
 #include "exact_sum.h"
+#include "krylov_device.h"
 #include "omodels_internal.h"
 
 namespace omodels {
-
-// ---------------------------------------------------------------------------
-// small dense block helpers (row-major, BS = 2 or 3)
-template <int BS, class S>
-__device__ __forceinline__ void bMatmul(const S* A, const S* B, S* C)
-{
-#pragma unroll
-    for (int i = 0; i < BS; ++i)
-#pragma unroll
-        for (int j = 0; j < BS; ++j) {
-            S s = A[i * BS] * B[j];
-#pragma unroll
-            for (int k = 1; k < BS; ++k) s += A[i * BS + k] * B[k * BS + j];
-            C[i * BS + j] = s;
-        }
-}
-
-template <int BS, class S>
-__device__ __forceinline__ bool bInvert(S* a)
-{
-    if (BS == 2) {
-        S det = a[0] * a[3] - a[1] * a[2];
-        if (!(det != S(0)) || !isfinite((double)det)) return false;
-        S r = S(1) / det;
-        S i00 = a[3] * r, i01 = -a[1] * r, i10 = -a[2] * r, i11 = a[0] * r;
-        a[0] = i00; a[1] = i01; a[2] = i10; a[3] = i11;
-        return true;
-    } else {
-        S c00 = a[4] * a[8] - a[5] * a[7];
-        S c01 = a[5] * a[6] - a[3] * a[8];
-        S c02 = a[3] * a[7] - a[4] * a[6];
-        S det = a[0] * c00 + a[1] * c01 + a[2] * c02;
-        if (!(det != S(0)) || !isfinite((double)det)) return false;
-        S r = S(1) / det;
-        S c10 = a[2] * a[7] - a[1] * a[8];
-        S c11 = a[0] * a[8] - a[2] * a[6];
-        S c12 = a[1] * a[6] - a[0] * a[7];
-        S c20 = a[1] * a[5] - a[2] * a[4];
-        S c21 = a[2] * a[3] - a[0] * a[5];
-        S c22 = a[0] * a[4] - a[1] * a[3];
-        a[0] = c00 * r; a[1] = c10 * r; a[2] = c20 * r;
-        a[3] = c01 * r; a[4] = c11 * r; a[5] = c21 * r;
-        a[6] = c02 * r; a[7] = c12 * r; a[8] = c22 * r;
-        return true;
-    }
-}
 
 // ---------------------------------------------------------------------------
 // SpMV: one thread per block row.
@@ -568,13 +524,6 @@ __device__ __forceinline__ double waveSum(double v)
     for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
     return v;
 }
-__device__ __forceinline__ double waveMax(double v)
-{
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_down(v, o, 64));
-    return v;
-}
-
 template <bool IsMax>
 __device__ __forceinline__ double blockReduce(double v)
 {
@@ -612,34 +561,6 @@ inline int dotBlocks(long m)
 {
     const long per = (long)kDotUnroll * kDotThreads;
     return (int)std::max(1L, std::min<long>(kDotMaxBlocks, (m + per - 1) / per));
-}
-
-__device__ __forceinline__ void markFail(KrylovScalars* ks, int tag)
-{
-    if (!ks->fail_code) { ks->fail_code = 2; ks->fail_tag = tag; }
-}
-
-// what the last workgroup does with the sums (s0, s1)
-__device__ __forceinline__ void dotEpilogue(int mode, double s0, double s1, KrylovScalars* ks, double eps, int tagOff,
-                                            double* out)
-{
-    if (mode == kDotValue) { *out = s0; return; }
-    const int tag = ks->tag_base + tagOff;
-    if (mode == kDotRho) {             // rho_i = <r0hat, r>, beta (bicgstabsolver.hh:197-206)
-        ks->rho_i = s0;
-        if (fabs(ks->rho) <= eps || fabs(ks->omega) <= eps) markFail(ks, tag);
-        ks->beta = (s0 / ks->rho) * (ks->alpha / ks->omega);
-        ks->rho = s0;
-    } else if (mode == kDotAlpha) {    // denom = <r0hat, v>, alpha (:230-236)
-        ks->denom = s0;
-        if (fabs(s0) <= eps) markFail(ks, tag);
-        ks->alpha = ks->rho / s0;
-        if (fabs(ks->alpha) <= eps) markFail(ks, tag);
-    } else {                           // omega = <t, s> / <t, t> (:287-292)
-        if (fabs(s0) <= eps) markFail(ks, tag);
-        ks->omega = s1 / s0;
-        if (fabs(ks->omega) <= eps) markFail(ks, tag);
-    }
 }
 
 // 16 bytes of a vector at the alignment of its scalar (a caller's own vector
@@ -728,28 +649,6 @@ void launchScalarProduct(long m, const double* x, const double* y, DotScratch* s
 {
     hipLaunchKernelGGL((k_xdot<double, 1>), dim3(dotBlocks(m)), dim3(kDotThreads), 0, st, m, x, y, sc,
                        (KrylovScalars*)nullptr, (int)kDotValue, 0.0, 0, out);
-}
-
-// the test after the first half of iteration tag_base / 2 (bicgstabsolver.hh:
-// 252-273) with the outcome of the previous second half (:286-318), in the
-// order of the host loop; once it ends the solve, the queued kernels of
-// the next iteration return at once
-__device__ __forceinline__ void criterion(double mx, bool change, KrylovScalars* ks)
-{
-    ks->resnorm = mx;
-    ks->stag_half = change ? 0 : 1;
-    const int tag = ks->tag_base;
-    int rc = -1, back = 0;
-    if (tag > 0 && ks->fail_code && ks->fail_tag == tag - 1) { rc = 2; back = 1; }
-    else if (tag > 0 && ks->stag_full_tag == tag - 1) { rc = 1; back = 1; }
-    else if (ks->fail_code) rc = 2;
-    else if (mx / fmax(1e-20, ks->init_norm) <= ks->tol || mx <= ks->abs_tol) rc = 0;
-    else if (ks->stag_half || mx > ks->max_error) rc = 1;
-    if (rc >= 0) {
-        ks->stop_rc = rc;
-        ks->stop_back = back;
-        ks->run = 0;
-    }
 }
 
 // The iterate's updates: one element-wise pass each, bounded by the memory

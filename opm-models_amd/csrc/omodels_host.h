@@ -289,6 +289,7 @@ private:
     template <class S> void spmvInner(const S* A, const S* x, S* y, const int* run);
     // a 3x3 system on the model's nx x ny x nz grid (7-point pattern)
     bool structured() const;
+    bool small_ = false;         // the whole solve in one launch (small_solve.h)
     bool prepared_ = false;
     bool tuned_ = false;
 };

@@ -211,7 +211,7 @@ struct KrylovScalars {
     int stag_half;        // change indicator all zero at the last half-step check
     int stag_full_tag;    // half-iteration index of a full-step stagnation, -1 if none
     int tag_base;         // half-iteration index of the current iteration's first half (2 it)
-    int pad_;
+    int iters;            // iterations of a solve that runs in one launch
     // the test after each first half, evaluated on the device so that the next
     // iteration can be queued before the host has seen this one's result
     double tol, abs_tol, max_error;
@@ -240,14 +240,23 @@ struct LevelSchedule {
     int nLevels = 0;
     std::vector<int> ptrHost;     // [nLevels+1]
     DevBuf<int> rows;             // rows ordered by level
+    // systems small enough for one workgroup (small_solve.h): the rows in
+    // chunks of one wave each, {row, its first entry, entries below | above
+    // the diagonal << 16, level} (row -1 in the unused slots of a chunk), with
+    // kSlotPad empty chunks of levels -1 and nLevels before and after them
+    static constexpr int kSlotPad = 48;
+    int nChunks = 0;
+    DevBuf<int4> slots;
+    // order: the rows by level (ptrHost is set); rp, diag: the pattern
+    void setRows(const std::vector<int>& order, int bs, const int* rp, const int* diag, hipStream_t s);
 };
 // the levels of a block pattern's rows for the triangular sweeps: a row's
 // level is one more than the largest level of the lower-numbered rows it is
 // coupled with in either direction, so the forward sweep (levels ascending)
 // and the backward sweep (descending) find every row they read done also
 // when the pattern is not symmetric
-void buildLevelSchedule(long rows, const std::vector<int>& rowPtr, const std::vector<int>& colIdx,
-                        LevelSchedule& L, hipStream_t s);
+void buildLevelSchedule(long rows, int bs, const std::vector<int>& rowPtr, const std::vector<int>& colIdx,
+                        const std::vector<int>& diag, LevelSchedule& L, hipStream_t s);
 void launchAddAuxiliary(int nb, const int* blockOff, const double* blocks, int nr, const int* resRow,
                         const double* resVals, double* jac, double* res, hipStream_t s);
 void launchAuxUpdate(long n, double* x, const double* delta, int* counters, hipStream_t s);
