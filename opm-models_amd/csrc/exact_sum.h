@@ -319,21 +319,27 @@ __device__ __forceinline__ bool lastToFinish(unsigned* ticket, int nBlocks, unsi
     return sMeta[1] != 0u;
 }
 
-// The same for a whole grid: many workgroups meet in kFinishGroups groups
-// first, whose tickets lie in lines of their own.  Atomics on one word pass at
-// about 13 ns each, so 256 workgroups on one ticket take 3.3 us; the groups'
-// second round trip takes 1 us, which fewer than 64 workgroups would not win
-// back.
+// For one thread of each workgroup of a grid, its result acknowledged: true in
+// the last one.  Many workgroups meet in kFinishGroups groups first, whose
+// tickets lie in lines of their own.  Atomics on one word pass at about 13 ns
+// each, so 256 workgroups on one ticket take 3.3 us; the groups' second round
+// trip takes 1 us, which fewer than 64 workgroups would not win back.  The
+// last one resets the tickets.
 constexpr int kFinishGroups = 16, kFinishFlat = 64;
 struct alignas(128) FinishTicket {
     unsigned n;
 };
+__device__ __forceinline__ bool takeTicket(FinishTicket* t, int count)
+{
+    if (__hip_atomic_fetch_add(&t->n, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != (unsigned)count - 1u) return false;
+    __hip_atomic_store(&t->n, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return true;
+}
 // tickets: kFinishGroups + 1, the last one the groups' own
-__device__ __forceinline__ bool lastOfGrid(FinishTicket* tickets, unsigned* sMeta)
+__device__ __forceinline__ bool lastTicketOfGrid(FinishTicket* tickets)
 {
     const int nb = (int)gridDim.x, G = nb > kFinishFlat ? kFinishGroups : 1, g = (int)blockIdx.x % G;
-    if (!lastToFinish(&tickets[g].n, (nb - g + G - 1) / G, sMeta)) return false;
-    return G == 1 || lastToFinish(&tickets[kFinishGroups].n, G, sMeta);
+    return takeTicket(&tickets[g], (nb - g + G - 1) / G) && (G == 1 || takeTicket(&tickets[kFinishGroups], G));
 }
 
 // exactRound by one wave: lane j holds limb j as a signed integer, and limbs

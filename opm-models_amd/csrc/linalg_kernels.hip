@@ -655,6 +655,8 @@ void launchScalarProduct(long m, const double* x, const double* y, DotScratch* s
 // (48 bytes an FP64 entry) or, on small systems, by the launch.  The maximum
 // and the change indicator of the workgroups are joined, and the test
 // evaluated, by the workgroup that finishes last: no second launch for them.
+// x and r by entries, FP64 / FP32, us (with a test launch of their own before):
+// 1440 3.3 / 3.5 (7.6 / 7.5), 400k 7.8 / 6.7 (9.1 / 8.1), 1.5M 15.0 / 9.8 (17.7 / 9.8).
 constexpr int kUpdThreads = 1024;
 constexpr int kUpdBlocks = kDotMaxBlocks;     // one workgroup per CU
 
@@ -664,12 +666,11 @@ inline int updateBlocks(long m, int perThread)
     return (int)std::max(1L, std::min<long>(kUpdBlocks, (m + per - 1) / per));
 }
 
-// f(i0, n): entries i0 .. i0 + n - 1 (n <= V, a compile-time V for full ones)
-template <int V, class F>
-__device__ __forceinline__ void forEntries(long m, F f)
+// entries of the piece at i (V, or fewer at the end, or none)
+template <int V>
+__device__ __forceinline__ int pieceLength(long m, long i)
 {
-    const long step = (long)gridDim.x * kUpdThreads * V;
-    for (long i = ((long)blockIdx.x * kUpdThreads + threadIdx.x) * V; i < m; i += step) f(i, (int)min((long)V, m - i));
+    return i + V <= m ? V : (i < m ? (int)(m - i) : 0);
 }
 
 template <int V, class S>
@@ -701,61 +702,70 @@ __device__ __forceinline__ void storeEntries(S* p, long i, int n, const S (&x)[V
 
 // p = r + (-beta) * (v*omega - p)   (bicgstabsolver.hh:211-222)
 template <class S>
-__global__ __launch_bounds__(kUpdThreads) void k_update_p(long m, const S* __restrict__ r, const S* __restrict__ v,
+__global__ __launch_bounds__(256) void k_update_p(long m, const S* __restrict__ r, const S* __restrict__ v,
     S* __restrict__ p, const KrylovScalars* __restrict__ ks)
 {
-    if (!ks->run) return;
     constexpr int V = Vec16<S>::kN;
+    const long i = ((long)blockIdx.x * 256 + threadIdx.x) * V;
+    if (i >= m || !ks->run) return;
+    const int n = pieceLength<V>(m, i);
     const S omega = (S)ks->omega, beta = (S)ks->beta;
-    forEntries<V>(m, [&](long i, int n) {
-        S rv[V], vv[V], pv[V];
-        loadEntries<V>(v, i, n, vv); loadEntries<V>(p, i, n, pv); loadEntries<V>(r, i, n, rv);
+    S rv[V], vv[V], pv[V];
+    loadEntries<V>(v, i, n, vv); loadEntries<V>(p, i, n, pv); loadEntries<V>(r, i, n, rv);
 #pragma unroll
-        for (int q = 0; q < V; ++q) {
-            S tmp = vv[q];
-            tmp *= omega;
-            tmp -= pv[q];
-            tmp *= -beta;
-            S pn = rv[q];
-            pn += tmp;
-            pv[q] = pn;
-        }
-        storeEntries<V>(p, i, n, pv);
-    });
+    for (int q = 0; q < V; ++q) {
+        S tmp = vv[q];
+        tmp *= omega;
+        tmp -= pv[q];
+        tmp *= -beta;
+        S pn = rv[q];
+        pn += tmp;
+        pv[q] = pn;
+    }
+    storeEntries<V>(p, i, n, pv);
 }
 template <class S>
 void launchUpdateP(long m, const S* r, const S* v, S* p, const KrylovScalars* ks, hipStream_t st)
 {
-    hipLaunchKernelGGL((k_update_p<S>), dim3(updateBlocks(m, Vec16<S>::kN)), dim3(kUpdThreads), 0, st, m, r, v, p, ks);
+    const long per = 256L * Vec16<S>::kN;
+    hipLaunchKernelGGL((k_update_p<S>), dim3((unsigned)((m + per - 1) / per)), dim3(256), 0, st, m, r, v, p, ks);
 }
 template void launchUpdateP<double>(long, const double*, const double*, double*, const KrylovScalars*, hipStream_t);
 template void launchUpdateP<float>(long, const float*, const float*, float*, const KrylovScalars*, hipStream_t);
 
 // Joins the workgroups' maximum and change indicator; true in thread 0 of the
-// last workgroup, which then has both over all entries.
-__device__ __forceinline__ bool joinUpdate(DotScratch* sc, double& mx, bool& change)
+// last workgroup, which then has both over all entries.  store() writes the
+// thread's last entries: after the workgroup's own result has gone out, so
+// that the wait for that result's acknowledgement is not behind them.
+template <class F>
+__device__ __forceinline__ bool joinUpdate(DotScratch* sc, double& mx, bool& change, F store)
 {
     constexpr int nw = kUpdThreads / 64;
     __shared__ double sMx[nw];
-    __shared__ unsigned sMeta[2], sAny[nw];
+    __shared__ unsigned sLast, sAny[nw];
     const int lane = (int)(threadIdx.x & 63u), w = (int)(threadIdx.x >> 6);
     mx = waveMax(mx);
     const bool any = __ballot(change) != 0ull;
     if (lane == 0) { sMx[w] = mx; sAny[w] = any ? 1u : 0u; }
     __syncthreads();
+    const int nb = (int)gridDim.x;
     if (w == 0) {
         mx = waveMax(lane < nw ? sMx[lane] : 0.0);
         change = __ballot(lane < nw && sAny[lane]) != 0ull;
-        if (gridDim.x == 1) return lane == 0;
-        if (lane == 0) {
+        if (lane == 0 && nb > 1) {
             __hip_atomic_store(&sc->blockMax[blockIdx.x], mx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __hip_atomic_store(&sc->blockAny[blockIdx.x], change ? 1u : 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __builtin_amdgcn_s_waitcnt(0x0F70);
+            sLast = lastTicketOfGrid(sc->updTicket) ? 1u : 0u;
         }
     }
-    if (gridDim.x == 1 || !lastOfGrid(sc->updTicket, sMeta) || w != 0) return false;
+    store();
+    if (nb == 1) return threadIdx.x == 0;
+    __syncthreads();
+    if (!sLast || w != 0) return false;
     mx = 0.0;
     unsigned a = 0u;
-    for (int k = lane; k < (int)gridDim.x; k += 64) {
+    for (int k = lane; k < nb; k += 64) {
         mx = fmax(mx, __hip_atomic_load(&sc->blockMax[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
         a |= __hip_atomic_load(&sc->blockAny[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
@@ -774,8 +784,12 @@ __global__ __launch_bounds__(kUpdThreads) void k_update_xr(long m, const S* __re
     const S alpha = (S)ks->alpha;
     double mx = 0.0;
     bool change = false;
-    forEntries<V>(m, [&](long i, int n) {
-        S yv[V], vv[V], xv[V], rv[V];
+    const long step = (long)gridDim.x * kUpdThreads * V;
+    long i = ((long)blockIdx.x * kUpdThreads + threadIdx.x) * V;
+    S xv[V], rv[V];
+    for (;; i += step) {
+        const int n = pieceLength<V>(m, i);
+        S yv[V], vv[V];
         loadEntries<V>(y, i, n, yv); loadEntries<V>(x, i, n, xv);
         loadEntries<V>(v, i, n, vv); loadEntries<V>(r, i, n, rv);
 #pragma unroll
@@ -792,9 +806,14 @@ __global__ __launch_bounds__(kUpdThreads) void k_update_xr(long m, const S* __re
                 change |= yv[q] != S(0);
             }
         }
+        if (i + step >= m) break;
         storeEntries<V>(x, i, n, xv); storeEntries<V>(r, i, n, rv);
-    });
-    if (joinUpdate(sc, mx, change)) criterion(mx, change, ks);
+    }
+    auto store = [&]() {
+        const int n = pieceLength<V>(m, i);
+        storeEntries<V>(x, i, n, xv); storeEntries<V>(r, i, n, rv);
+    };
+    if (joinUpdate(sc, mx, change, store)) criterion(mx, change, ks);
 }
 
 template <class S>
@@ -826,8 +845,12 @@ __global__ __launch_bounds__(kUpdThreads) void k_update_xr2(long m, const S* __r
     const S omega = (S)ks->omega;
     double mx = 0.0;
     bool change = false;
-    forEntries<V>(m, [&](long i, int n) {
-        S zv[V], tv[V], xv[V], rv[V];
+    const long step = (long)gridDim.x * kUpdThreads * V;
+    long i = ((long)blockIdx.x * kUpdThreads + threadIdx.x) * V;
+    S xv[V], rv[V];
+    for (;; i += step) {
+        const int n = pieceLength<V>(m, i);
+        S zv[V], tv[V];
         loadEntries<V>(z, i, n, zv); loadEntries<V>(x, i, n, xv);
         loadEntries<V>(t, i, n, tv); loadEntries<V>(r, i, n, rv);
 #pragma unroll
@@ -836,9 +859,14 @@ __global__ __launch_bounds__(kUpdThreads) void k_update_xr2(long m, const S* __r
             if (q < n) change |= zv[q] != S(0);
             rv[q] += -omega * tv[q];
         }
+        if (i + step >= m) break;
         storeEntries<V>(x, i, n, xv); storeEntries<V>(r, i, n, rv);
-    });
-    if (!joinUpdate(sc, mx, change)) return;
+    }
+    auto store = [&]() {
+        const int n = pieceLength<V>(m, i);
+        storeEntries<V>(x, i, n, xv); storeEntries<V>(r, i, n, rv);
+    };
+    if (!joinUpdate(sc, mx, change, store)) return;
     if (!change && ks->stag_full_tag < 0) ks->stag_full_tag = ks->tag_base + tagOff;
     ks->tag_base += advance;
 }
