@@ -107,21 +107,39 @@ def test_simulate_matches_oracle(precision, solver_float):
     assert mass == pytest.approx(pg.inflow_rate * 1.0 * 3000.0, rel=1e-7)
 
 
+def _run(dims, t_end, **kw):
+    m = om.LensModel(om.lens_problem(nx=dims[0], ny=dims[1]))
+    rc, th, dth, log, st = m.simulate(om.default_params(newton_tol=1e-8, **kw), t_end, 250.0)
+    assert rc == 0
+    return m.get_solution(), dth, [r[3] for r in log], st.linear_iters
+
+
+def _assert_same_run(a, b):
+    assert a[3] == b[3] and a[2] == b[2]
+    assert np.array_equal(a[1], b[1])
+    assert np.array_equal(a[0].view(np.uint64), b[0].view(np.uint64))
+
+
 @pytest.mark.parametrize("precision", [0, 2])
-def test_graph_run_is_identical_to_eager(precision):
+@pytest.mark.parametrize("dims,schedule,t_end", [((48, 32), 0, 3000.0), ((48, 32), 1, 3000.0), ((91, 91), 0, 250.0)])
+def test_graph_run_is_identical_to_eager(dims, schedule, t_end, precision):
     """The lens run with its BiCGStab iterations replayed from graphs matches
-    the eager run bit for bit."""
-    pg, _ = problems()
-    out = []
-    for g in (0, 1):
-        m = om.LensModel(pg)
-        rc, th, dth, log, st = m.simulate(om.default_params(newton_tol=1e-8, precision=precision, graph=g),
-                                          3000.0, 250.0)
-        assert rc == 0
-        out.append((m.get_solution(), dth, st.linear_iters))
-    assert out[0][2] == out[1][2]
-    assert np.array_equal(out[0][1], out[1][1])
-    assert np.array_equal(out[0][0].view(np.uint64), out[1][0].view(np.uint64))
+    the eager run bit for bit: by level-scheduled launches on any grid
+    (ilu_schedule = 1), and where the default takes them, above 8192 cells.
+    At 48x32 the default is one launch per solve, which has no iteration to
+    record: there the switch must change nothing."""
+    _assert_same_run(_run(dims, t_end, precision=precision, ilu_schedule=schedule, graph=0),
+                     _run(dims, t_end, precision=precision, ilu_schedule=schedule, graph=1))
+
+
+@pytest.mark.parametrize("precision", [0, 2])
+@pytest.mark.parametrize("dims,t_end", [((2, 1), 500.0), ((7, 5), 500.0), ((48, 32), 1000.0), ((128, 64), 250.0)])
+def test_one_workgroup_solve_is_identical_to_launches(dims, t_end, precision):
+    """The 2x2 one-workgroup factorization and solve against the
+    level-scheduled launches, bit for bit with the same iteration counts, up to
+    8192 cells: the most whose vector fits the workgroup's LDS."""
+    _assert_same_run(_run(dims, t_end, precision=precision, ilu_schedule=0),
+                     _run(dims, t_end, precision=precision, ilu_schedule=1))
 
 
 @pytest.mark.parametrize("precision,solver_float,tol", [(0, 0, 1e-10), (2, 1, 1e-8)])
