@@ -6,6 +6,7 @@
 // Instances whose solve has finished are masked by their `active` flag.
 #include "ensemble.h"
 #include "ens_ops.h"
+#include "krylov_device.h"
 
 namespace omodels {
 
@@ -17,46 +18,27 @@ template <class S> __device__ __forceinline__ S* vec(const EnsInst& I, int id);
 template <> __device__ __forceinline__ double* vec<double>(const EnsInst& I, int id) { return I.dv[id]; }
 template <> __device__ __forceinline__ float* vec<float>(const EnsInst& I, int id) { return I.fv[id]; }
 
-__device__ __forceinline__ double waveSum(double v)
-{
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-    return v;
-}
-__device__ __forceinline__ double waveMax(double v)
-{
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_down(v, o, 64));
-    return v;
-}
-template <bool IsMax>
-__device__ __forceinline__ double blockReduce(double v)
+__device__ __forceinline__ double blockMax(double v)
 {
     __shared__ double sm[kT / 64];
-    v = IsMax ? waveMax(v) : waveSum(v);
+    v = waveMax(v);
     const int w = threadIdx.x / 64, l = threadIdx.x % 64;
     if (l == 0) sm[w] = v;
     __syncthreads();
     double r = 0.0;
     if (threadIdx.x == 0) {
         r = sm[0];
-        for (int q = 1; q < kT / 64; ++q) r = IsMax ? fmax(r, sm[q]) : r + sm[q];
+        for (int q = 1; q < kT / 64; ++q) r = fmax(r, sm[q]);
     }
     __syncthreads();
     return r;
 }
-// sum / max of the partials of instance b (chunks [first[b], first[b+1]))
-template <bool IsMax>
-__device__ __forceinline__ double instReduce(const double* __restrict__ part, int c0, int c1)
+// max of the partials of instance b (chunks [first[b], first[b+1]))
+__device__ __forceinline__ double instMax(const double* __restrict__ part, int c0, int c1)
 {
     double v = 0.0;
-    for (int k = c0 + (int)threadIdx.x; k < c1; k += kT) v = IsMax ? fmax(v, part[k]) : v + part[k];
-    return blockReduce<IsMax>(v);
-}
-
-__device__ __forceinline__ void markFail(KrylovScalars* ks, int tag)
-{
-    if (!ks->fail_code) { ks->fail_code = 2; ks->fail_tag = tag; }
+    for (int k = c0 + (int)threadIdx.x; k < c1; k += kT) v = fmax(v, part[k]);
+    return blockMax(v);
 }
 
 }  // namespace
@@ -96,7 +78,7 @@ __global__ __launch_bounds__(kT) void k_e_xdot(const EnsInst* __restrict__ insts
     if (!act[it.x]) return;
     constexpr int nw = kT / 64;
     __shared__ unsigned long long sAcc[NACC * kAccLimbs];
-    __shared__ unsigned sMeta[5];
+    __shared__ unsigned sMeta[2];
     clearLimbs(sAcc, NACC, sMeta);
     __syncthreads();
     const EnsInst& I = insts[it.x];
@@ -210,8 +192,8 @@ __global__ __launch_bounds__(kT) void k_e_update_xr(const EnsInst* __restrict__ 
             if (yi != S(0)) nz = 1.0;
         }
     }
-    mx = blockReduce<true>(mx);
-    nz = blockReduce<true>(nz);
+    mx = blockMax(mx);
+    nz = blockMax(nz);
     if (threadIdx.x == 0) { part[blockIdx.x] = mx; part[nChunks + blockIdx.x] = nz; }
 }
 
@@ -220,8 +202,8 @@ __global__ __launch_bounds__(kT) void k_e_crit_final(const int* __restrict__ fir
 {
     const int b = blockIdx.x;
     if (!act[b]) return;
-    const double mx = instReduce<true>(part, first[b], first[b + 1]);
-    const double nz = instReduce<true>(part + nChunks, first[b], first[b + 1]);
+    const double mx = instMax(part, first[b], first[b + 1]);
+    const double nz = instMax(part + nChunks, first[b], first[b + 1]);
     if (threadIdx.x != 0) return;
     ksAll[b].resnorm = mx;
     ksAll[b].stag_half = nz == 0.0 ? 1 : 0;
@@ -253,7 +235,7 @@ __global__ __launch_bounds__(kT) void k_e_update_xr2(const EnsInst* __restrict__
             r[i] += -omega * y[i];
         }
     }
-    nz = blockReduce<true>(nz);
+    nz = blockMax(nz);
     if (threadIdx.x == 0) part[blockIdx.x] = nz;
 }
 
@@ -265,7 +247,7 @@ __global__ __launch_bounds__(kT) void k_e_stag_final(const int* __restrict__ fir
 {
     const int b = blockIdx.x;
     if (!act[b]) return;
-    const double nz = instReduce<true>(part, first[b], first[b + 1]);
+    const double nz = instMax(part, first[b], first[b + 1]);
     if (threadIdx.x != 0) return;
     if (nz == 0.0 && ksAll[b].stag_full_tag < 0) ksAll[b].stag_full_tag = ksAll[b].tag_base + tagOff;
     ksAll[b].tag_base += 2;
@@ -341,7 +323,7 @@ __global__ __launch_bounds__(kT) void k_e_maxabs_partial(const EnsInst* __restri
 #pragma unroll
         for (int e = 0; e < 3; ++e) mx = fmax(mx, fabs((double)x[3 * c + e]));
     }
-    mx = blockReduce<true>(mx);
+    mx = blockMax(mx);
     if (threadIdx.x == 0) part[blockIdx.x] = mx;
 }
 __global__ __launch_bounds__(kT) void k_e_max_final(const int* __restrict__ first, const int* __restrict__ act,
@@ -349,7 +331,7 @@ __global__ __launch_bounds__(kT) void k_e_max_final(const int* __restrict__ firs
 {
     const int b = blockIdx.x;
     if (!act[b]) return;
-    const double mx = instReduce<true>(part, first[b], first[b + 1]);
+    const double mx = instMax(part, first[b], first[b + 1]);
     if (threadIdx.x == 0) out[b] = mx;
 }
 

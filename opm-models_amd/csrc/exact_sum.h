@@ -279,7 +279,7 @@ __device__ __forceinline__ void accumulateBands(const double (&p)[U], unsigned l
 }
 
 // The workgroup's limbs of nAcc sums (LDS, nAcc * kAccLimbs) and their flags
-// (3 bits each) in sMeta[0]; sMeta[1..4] scratch.
+// (3 bits each) in sMeta[0]; sMeta[1] belongs to lastToFinish.
 __device__ __forceinline__ void clearLimbs(unsigned long long* sAcc, int nAcc, unsigned* sMeta)
 {
     for (int t = (int)threadIdx.x; t < nAcc * kAccLimbs; t += (int)blockDim.x) sAcc[t] = 0ull;

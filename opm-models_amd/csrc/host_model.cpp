@@ -104,7 +104,7 @@ void LinearSystem::initSystem(hipStream_t s)
     if (hipGetDevice(&dev) != hipSuccess) throw std::runtime_error("no HIP device available");
     if (s) stream = s;
     else { OM_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking)); ownStream = true; }
-    partial.alloc(2 * kRedBlocks);
+    partial.alloc(kRedBlocks);
     dots.alloc(1);
     OM_HIP(hipMemsetAsync(dots.p, 0, sizeof(DotScratch), stream));
     scal.alloc(8);

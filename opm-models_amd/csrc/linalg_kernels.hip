@@ -8,8 +8,9 @@
 //   BiCGStab vector steps    BiCGStabSolver::apply (bicgstabsolver.hh:120-330)
 //   CombinedCriterion norms  combinedcriterion.hh:54-236
 //
-// Reductions use a fixed number of partial sums and a fixed tree, so results
-// are reproducible run to run; BiCGStab scalars stay in device memory.
+// Sums are exact (exact_sum.h) and the other reductions maxima, so results do
+// not depend on the order of the workgroups; BiCGStab scalars stay in device
+// memory.
 #include <hipcub/hipcub.hpp>
 
 #include "block_ops.h"
@@ -515,39 +516,31 @@ template void launchJacobiSweeps<float>(int, int, const int*, const int*, const 
                                         float*, float*, double, const int*, hipStream_t);
 
 // ---------------------------------------------------------------------------
-// Reductions: kRedBlocks fixed partials of 256 threads, then one block.
+// Maximum norms: kRedBlocks partials of 256 threads, then one block.
 constexpr int kRedThreads = 256;
 
-__device__ __forceinline__ double waveSum(double v)
-{
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-    return v;
-}
-template <bool IsMax>
-__device__ __forceinline__ double blockReduce(double v)
+__device__ __forceinline__ double blockMax(double v)
 {
     __shared__ double sm[kRedThreads / 64];
-    v = IsMax ? waveMax(v) : waveSum(v);
+    v = waveMax(v);
     const int w = threadIdx.x / 64, l = threadIdx.x % 64;
     if (l == 0) sm[w] = v;
     __syncthreads();
     double r = 0.0;
     if (threadIdx.x == 0) {
         r = sm[0];
-        for (int q = 1; q < kRedThreads / 64; ++q) r = IsMax ? fmax(r, sm[q]) : r + sm[q];
+        for (int q = 1; q < kRedThreads / 64; ++q) r = fmax(r, sm[q]);
     }
     __syncthreads();
     return r;
 }
 
-// final reduce of kRedBlocks partials with one block of kRedThreads
-template <bool IsMax>
-__device__ __forceinline__ double finalReduce(const double* __restrict__ partial)
+// the maximum of kRedBlocks partials with one block of kRedThreads
+__device__ __forceinline__ double finalMax(const double* __restrict__ partial)
 {
-    double v = IsMax ? 0.0 : 0.0;
-    for (int k = threadIdx.x; k < kRedBlocks; k += kRedThreads) v = IsMax ? fmax(v, partial[k]) : v + partial[k];
-    return blockReduce<IsMax>(v);
+    double v = 0.0;
+    for (int k = threadIdx.x; k < kRedBlocks; k += kRedThreads) v = fmax(v, partial[k]);
+    return blockMax(v);
 }
 
 // Scalar products: the exact sum of the products, rounded once (exact_sum.h),
@@ -586,7 +579,7 @@ __global__ __launch_bounds__(kDotThreads) void k_xdot(long m, const S* __restric
     if (ks && !ks->run) return;
     constexpr int nw = kDotThreads / 64, V = Vec16<S>::kN;
     __shared__ unsigned long long sAcc[NACC * kAccLimbs];
-    __shared__ unsigned sMeta[5];
+    __shared__ unsigned sMeta[2];
     clearLimbs(sAcc, NACC, sMeta);
     __syncthreads();
     const int lane = (int)(threadIdx.x & 63u);
@@ -887,12 +880,12 @@ __global__ __launch_bounds__(kRedThreads) void k_maxabs_partial(long m, const S*
     double mx = 0.0;
     for (long i = (long)blockIdx.x * kRedThreads + threadIdx.x; i < m; i += (long)kRedBlocks * kRedThreads)
         mx = fmax(mx, fabs((double)x[i]));
-    mx = blockReduce<true>(mx);
+    mx = blockMax(mx);
     if (threadIdx.x == 0) part[blockIdx.x] = mx;
 }
 __global__ __launch_bounds__(kRedThreads) void k_max_final(const double* __restrict__ part, double* out)
 {
-    const double mx = finalReduce<true>(part);
+    const double mx = finalMax(part);
     if (threadIdx.x == 0) *out = mx;
 }
 template <class S>

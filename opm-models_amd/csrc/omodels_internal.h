@@ -221,7 +221,7 @@ struct KrylovScalars {
     int pad2_;
 };
 
-constexpr int kRedBlocks = 1024;     // partial sums per reduction (fixed => deterministic)
+constexpr int kRedBlocks = 1024;     // partial maxima per norm
 
 // run: nullptr, or a device flag; the product is skipped while it is 0
 template <class S> void launchSpmv(int n, int bs, const int* rp, const int* ci, const S* a,

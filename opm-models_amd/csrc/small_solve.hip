@@ -326,8 +326,8 @@ __global__ __launch_bounds__(kThreads) void k_small_bicgstab(SmallArgs<S> a)
         smallDot<S, 1>(m, a.b, a.r, sh, kDotRho, eps, 0);
         {
             const S omega = (S)ks.omega, beta = (S)ks.beta;
-        #pragma unroll 1
-    for (int i = tid; i < m; i += kThreads) {
+#pragma unroll 1
+            for (int i = tid; i < m; i += kThreads) {
                 S tmp = a.v[i];
                 tmp *= omega;
                 tmp -= a.p[i];
@@ -346,8 +346,8 @@ __global__ __launch_bounds__(kThreads) void k_small_bicgstab(SmallArgs<S> a)
             const S alpha = (S)ks.alpha;
             mx = 0.0;
             change = false;
-        #pragma unroll 1
-    for (int i = tid; i < m; i += kThreads) {
+#pragma unroll 1
+            for (int i = tid; i < m; i += kThreads) {
                 const S yi = sv[i];
                 S tmp = yi;
                 tmp *= alpha;
@@ -379,8 +379,8 @@ __global__ __launch_bounds__(kThreads) void k_small_bicgstab(SmallArgs<S> a)
             const S omega = (S)ks.omega;
             change = false;
             mx = 0.0;
-        #pragma unroll 1
-    for (int i = tid; i < m; i += kThreads) {
+#pragma unroll 1
+            for (int i = tid; i < m; i += kThreads) {
                 const S zi = sv[i];
                 a.x[i] += omega * zi;
                 change |= zi != S(0);
