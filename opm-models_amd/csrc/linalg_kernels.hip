@@ -568,10 +568,12 @@ struct __attribute__((packed, aligned(sizeof(S)))) Vec16 {
 // Small products are bounded by latency (the launch, one pass, the limbs'
 // and the ticket's atomics, the rounding), large ones by the loads: each wave
 // takes kDotUnroll * 64 consecutive entries per pass in 16-byte loads and
-// issues the next pass's before it splits this one's products.  FP64, us by
-// entries (before: 8-byte loads, one thread rounding):
-//   NACC 1: 1440 5.4 (8.2), 400k 6.8 (9.9), 1.5M 9.3 (13.4), 6M 20.5 (36.6);
-//   NACC 2: 1440 7.2 (13.1), 400k 8.8 (15.3), 1.5M 13.2 (23.0).
+// issues the next pass's before it splits this one's products.  us (before:
+// 8-byte loads, one thread rounding), one sum / two sums inside a solve:
+//   FP64 1.3M entries 12.4 (19.9) / 16.7 (28.1), 1.5M 13.3 (20.1) / 18.1 (30.5);
+//   FP32 1.5M 10.4 (16.5) / 14.6 (24.8), 6M 21.4 (42.2) / 34.1 (60.2);
+// omodels_scalar_product_noalloc back to back, which clears its scratch first:
+//   1440 8.5 (10.1), 400k 9.0 (12.1), 1.5M 11.3 (15.2), 6M 22.8 (37.6), 100M 274 (588).
 template <class S, int NACC>
 __global__ __launch_bounds__(kDotThreads) void k_xdot(long m, const S* __restrict__ a, const S* __restrict__ b,
     DotScratch* __restrict__ sc, KrylovScalars* ks, int mode, double eps, int tagOff, double* out)
@@ -648,8 +650,11 @@ void launchScalarProduct(long m, const double* x, const double* y, DotScratch* s
 // (48 bytes an FP64 entry) or, on small systems, by the launch.  The maximum
 // and the change indicator of the workgroups are joined, and the test
 // evaluated, by the workgroup that finishes last: no second launch for them.
-// x and r by entries, FP64 / FP32, us (with a test launch of their own before):
-// 1440 3.3 / 3.5 (7.6 / 7.5), 400k 7.8 / 6.7 (9.1 / 8.1), 1.5M 15.0 / 9.8 (17.7 / 9.8).
+// x and r by entries, us (with a test launch of their own before), back to
+// back FP64 / FP32: 1440 3.3 / 3.5 (7.6 / 7.5), 400k 7.8 / 6.7 (9.1 / 8.1), 1.5M
+// 15.0 / 9.8 (17.7 / 9.8).  Inside a solve, whose other kernels leave less of
+// the vectors in the caches: first half FP64 1.5M 18.4 (14.7 + 4.8), FP32 1.5M
+// 11.2 (8.0 + 5.0), 6M 28.1 (24.2 + 4.8); second half FP64 1.5M 16.0 (13.8 + 4.6).
 constexpr int kUpdThreads = 1024;
 constexpr int kUpdBlocks = kDotMaxBlocks;     // one workgroup per CU
 

@@ -4,7 +4,7 @@
 // exact accumulator in a file-scope device array instead of an allocation.
 //
 // `scratch` holds the exact sum's device accumulators and tickets (DotScratch,
-// 6.5 KiB) per GPU for the life of the process.  In host code its name is
+// 6.4 KiB) per GPU for the life of the process.  In host code its name is
 // only a stand-in; the device address of each GPU's copy is looked up once per
 // device with hipGetSymbolAddress and used for every launch.  All calls on one
 // GPU share it: calls that overlap on one GPU (two streams, two threads) race
