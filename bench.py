@@ -118,11 +118,14 @@ def amg_bytes(levels, pre=2, post=2, n=3, s=8):
     coarsest inverse are FP64).  Per level of N cells and NNZB blocks: a
     sweep reads the off-diagonal blocks, the inverted diagonal blocks, b and x
     and writes x (the first, from x = 0, reads only the blocks of neighbours
-    swept before a cell: half of the off-diagonal ones, and no x); the
-    residual reads the blocks, b and x and writes r; the restriction reads r;
-    the prolongation reads and writes x.  The coarsest level reads its dense
-    inverse.  Setup (FP64): every level's matrix read once (structured
-    layout, 7 slots), coarse matrices and inverted diagonal blocks written."""
+    swept before a cell, half of the off-diagonal ones, and the even cells' x);
+    the residual is formed on the even cells: half of the off-diagonal blocks,
+    the even cells' diagonal ones, b and r, and x; the restriction reads that r;
+    the first backward colour reads the coarse solution (without backward sweeps
+    the prolongation is a pass of its own, which reads and writes x).  The
+    coarsest level reads its dense inverse.  Setup (FP64): every level's matrix
+    read once (structured layout, 7 slots), coarse matrices and inverted
+    diagonal blocks written."""
     bb = n * n * s
     cyc = 0
     setup = 0
@@ -139,12 +142,14 @@ def amg_bytes(levels, pre=2, post=2, n=3, s=8):
         Nc = 1
         for q in levels[l + 1]:
             Nc *= q
-        zero_sweep = ((nnzb - N) // 2) * bb + piv + 2 * vec
+        even = (N + 1) // 2
+        half = (nnzb - N) // 2
+        zero_sweep = half * bb + piv + 2 * vec + n * s * even
         sweep = (nnzb - N) * bb + piv + 3 * vec
         cyc += zero_sweep + (pre - 1 + post) * sweep
-        cyc += nnzb * bb + 3 * vec                 # residual
-        cyc += vec + n * s * Nc                    # restriction
-        cyc += 2 * vec + n * s * Nc                # prolongation
+        cyc += (half + even) * bb + vec + 2 * n * s * even           # residual
+        cyc += n * s * even + n * s * Nc                             # restriction
+        cyc += n * s * Nc + (0 if post else 2 * vec)                 # correction
         setup += 7 * bb64 * N + piv + 7 * bb64 * Nc
     return cyc, setup
 
